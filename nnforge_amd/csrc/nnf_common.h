@@ -37,6 +37,17 @@ namespace nnf
 		return ctx;
 	}
 
+	// n / divisor with magic = ceil(2^32 / divisor), exact while n * divisor < 2^32
+	__device__ __forceinline__ uint32_t fast_divide(uint32_t n, uint32_t divisor, uint32_t magic)
+	{
+		return (divisor == 1) ? n : __umulhi(n, magic);
+	}
+
+	inline uint32_t magic_of(uint32_t divisor)
+	{
+		return (divisor >= 2) ? static_cast<uint32_t>(((1ull << 32) + divisor - 1) / divisor) : 0u; // fast_divide does not use it for 1
+	}
+
 	// Consecutive workgroups are handed to consecutive XCDs (eight dies, an L2 each). Work items that touch common memory -
 	// the bands of a plane: the input rows two of them stage, the output cache line two of them write - are `together`
 	// consecutive work items; of every 8 * together workgroups the ones with the same index modulo 8 take them, so that
@@ -212,6 +223,8 @@ namespace nnf
 		const nnf_hip_chain_desc* prologue, const float* const* chunk_ptrs, bool plan_only);
 	bool window2d_launch(hipStream_t stream, int op, float mult, float* output, const float* input, uint32_t input_total, uint32_t plane_count,
 		uint32_t in_w, uint32_t in_h, uint32_t out_w, uint32_t out_h, uint32_t win_w, uint32_t win_h, uint32_t stride_x, uint32_t stride_y);
+	bool window3d_launch(hipStream_t stream, int op, float mult, float* output, const float* input, uint32_t input_total, uint32_t plane_count,
+		const uint32_t (&in_size)[3], const uint32_t (&out_size)[3], const uint32_t (&window)[3], const uint32_t (&stride)[3]);
 	int feature_map_stat_init(hipStream_t stream, nnf_hip_running_stat* device_stats, uint32_t feature_map_count);
 	int feature_map_stat_workspace_bytes(uint32_t entry_count, uint32_t feature_map_count, uint32_t neuron_count_per_feature_map, size_t* bytes);
 	int feature_map_stat_partial_count(uint32_t entry_count, uint32_t feature_map_count, uint32_t neuron_count_per_feature_map,

@@ -16,12 +16,6 @@ namespace nnf
 	{
 		constexpr int prologue_block_size = 256; // lanes per workgroup of the kernels that apply a prologue
 
-		// n / divisor with magic = ceil(2^32 / divisor), exact while n * divisor < 2^32
-		__device__ __forceinline__ uint32_t fast_divide(uint32_t n, uint32_t divisor, uint32_t magic)
-		{
-			return (divisor == 1) ? n : __umulhi(n, magic);
-		}
-
 		constexpr uint32_t prologue_weighted_max = 2;  // layers with weights (batch norm, PReLU) a prologue may hold
 		constexpr uint32_t prologue_coef_floats = 768; // LDS a workgroup sets aside for its planes' coefficients
 		constexpr uint32_t prologue_planes_max = 256;  // one lane per plane fetches the weights
@@ -413,11 +407,6 @@ namespace nnf
 				}
 			}
 			apply_prologue<VECTORS, EXP, UNIFORM, SPLIT>(v, off, coef, own, pro, exp_ctx, arm1_end, pro.op_count, two);
-		}
-
-		uint32_t magic_of(uint32_t divisor)
-		{
-			return (divisor >= 2) ? static_cast<uint32_t>(((1ull << 32) + divisor - 1) / divisor) : 0u; // fast_divide does not use it for 1
 		}
 
 		// The layers of a single-input group without Add - or, with allow_join, of two inputs joined by an Add -

@@ -188,6 +188,46 @@ def test_max_subsampling(gpu, shape, windows, strides, round_ups, is_min):
     assert T.bit_mismatches(got, want) == 0
 
 
+# nnf_window3d.hip: results are bits, so nothing but equality will do
+VOLUME_CASES = [
+    # shape (x last), windows (x first), strides, round_ups
+    ((3, 2, 28, 28, 28), [2, 2, 2], None, None),                      # slices of one volume, pairs of outputs, bands of unequal depth
+    ((40, 30, 28, 28, 28), [2, 2, 2], None, None),                    # ... at the full staging size
+    ((1, 3, 9, 64, 64), [3, 3, 3], [2, 2, 2], [True, True, True]),    # rows and slices in bands, pairs whose last window is cut off
+    ((2, 3, 9, 53, 53), [2, 2, 2], None, None),                       # odd rows: runs that start anywhere inside a float4
+    ((1, 5, 17, 61, 59), [3, 3, 3], [2, 2, 2], [True, False, True]),
+    ((7, 11, 7, 7, 7), [3, 3, 3], [2, 2, 2], [True, True, True]),     # several volumes per workgroup, the last workgroup short
+    ((5, 3, 4, 6, 8), [2, 2, 2], None, None),
+    ((1, 1, 3, 3, 3), [2, 2, 2], [1, 1, 1], None),                    # 27 floats: the tensor's last values outside a float4
+    ((1, 1, 3, 33, 241), [2, 2, 2], [1, 2, 1], None),                 # ... in the last of several runs
+    ((2, 2, 12, 40, 31), [5, 2, 3], [3, 1, 2], [True, False, True]),  # run-time window sizes
+    ((1, 2, 6, 20, 700), [3, 3, 3], [3, 3, 3], None),
+    ((1, 1, 4, 3, 9000), [2, 2, 2], None, None),                      # not even one window's rows fit LDS: the general kernel
+]
+
+
+@pytest.mark.parametrize("is_min", [False, True])
+@pytest.mark.parametrize("shape,windows,strides,round_ups", VOLUME_CASES)
+def test_max_subsampling_of_volumes(gpu, shape, windows, strides, round_ups, is_min):
+    x = spiced(T.rng(68, sum(shape)), shape)
+    got = run_max_subsampling(gpu, x, windows, strides, round_ups, is_min=is_min)
+    want = oracle.max_subsampling(x, windows, strides=strides, round_ups=round_ups, is_min=is_min)
+    assert got.shape == want.shape
+    assert T.bit_mismatches(got, want) == 0
+
+
+@pytest.mark.parametrize("shape,windows", [((3, 2, 28, 28, 28), [2, 2, 2]), ((2, 3, 9, 53, 53), [3, 3, 3]), ((7, 11, 7, 9, 8), [2, 3, 1]), ((1, 1, 4, 3, 9000), [2, 2, 2])])
+def test_average_subsampling_of_volumes(gpu, shape, windows):
+    x = T.normal(T.rng(69, sum(shape)), shape)
+    mult = 1.0 / float(np.prod(windows))
+    want = oracle.average_subsampling(x, windows, mult=mult)
+    d_out = gpu.torch.full((want.size,), float("nan"), dtype=gpu.torch.float32, device=gpu.device)
+    rc = gpu.lib.nnf_hip_average_subsampling_nd_forward(gpu.stream, d_out.data_ptr(), gpu.to_device(x).data_ptr(), shape[0], shape[1], 3,
+                                                        u32(list(shape[2:])[::-1]), u32(windows), 1, 1, mult)
+    assert rc == 0, capi.error_string(rc)
+    assert T.bit_mismatches(gpu.to_host(d_out, want.shape), want) == 0
+
+
 @pytest.mark.parametrize("fm,en", [(3, 1), (1, 2), (2, 3)])
 def test_max_subsampling_over_feature_maps_and_entries(gpu, fm, en):
     x = spiced(T.rng(65, fm * 10 + en), (6, 12, 9, 10))
