@@ -339,7 +339,7 @@ NNF_HIP_API int nnf_hip_feature_map_stat_accumulate(void* stream, nnf_hip_runnin
  * NNF_HIP_STAT_STATIC_SCRATCH_BYTES / 32 = 8192 partial states, one per feature map and run of entries. The runs
  * are planned inside that limit; a shape is refused (NNF_HIP_ESCRATCH, nothing launched) only when even the longest
  * runs the kernels' index arithmetic allows leave more states than that: more than 8192 feature maps, or planes of
- * u loads (u = neuron_count_per_feature_map / 4, or neuron_count_per_feature_map when that is no multiple of 4) with
+ * u float4 loads (u = the most float4s a plane of neuron_count_per_feature_map floats can touch) with
  * feature_map_count * ceil(entry_count / max(1, floor((2^32 - 1) / u^2))) > 8192. All calls on one GPU share the
  * array: calls that can overlap (different streams, different threads) race on it and must be ordered by the
  * caller; nothing in it has to be cleared between calls (the first launch writes every state the second reads). */

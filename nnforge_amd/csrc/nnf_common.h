@@ -48,6 +48,23 @@ namespace nnf
 		return (divisor >= 2) ? static_cast<uint32_t>(((1ull << 32) + divisor - 1) / divisor) : 0u; // fast_divide does not use it for 1
 	}
 
+	// The value of another lane of the same row of 16: quad swaps 0xB1 (lane ^ 1) and 0x4E (lane ^ 2), row_half_mirror 0x141,
+	// row_mirror 0x140 - taken in this order they combine all 16 lanes.
+	template<int CTRL>
+	__device__ __forceinline__ float dpp_move(float v)
+	{
+		return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+	}
+
+	template<int CTRL>
+	__device__ __forceinline__ double dpp_move(double v)
+	{
+		const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+		const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(bits), CTRL, 0xF, 0xF, false));
+		const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(bits >> 32), CTRL, 0xF, 0xF, false));
+		return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+	}
+
 	// Consecutive workgroups are handed to consecutive XCDs (eight dies, an L2 each). Work items that touch common memory -
 	// the bands of a plane: the input rows two of them stage, the output cache line two of them write - are `together`
 	// consecutive work items; of every 8 * together workgroups the ones with the same index modulo 8 take them, so that

@@ -25,12 +25,6 @@ namespace nnf
 			return (a < b) ? b : a;
 		}
 
-		template<int CTRL>
-		__device__ __forceinline__ float dpp_move(float v)
-		{
-			return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-		}
-
 		__device__ __forceinline__ float read_lane(float v, int lane)
 		{
 			return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));

@@ -73,6 +73,11 @@ def check(got, want, scale):
     (1, 1, 100003),        # one long plane, not a multiple of 4: segments of single floats
     (3, 2, 16388),         # segments of unequal length
     (1000, 2, 4),          # many entries per run
+    (13, 37, 35, 35),      # planes that start anywhere inside a float4
+    (5, 3, 2),             # tensors that end inside a float4: the last values belong to several planes
+    (2, 1, 3), (1, 3, 1),
+    (1, 1, 24577), (1, 2, 32770), (1, 1, 32771),   # ... to the last segment of a plane, or the one before it
+    (300, 5, 11),          # more than 64 runs' worth of entries per feature map
 ])
 def test_statistics_match_the_sequential_update(gpu, shape):
     gen = T.rng(70, sum(shape))
