@@ -242,11 +242,24 @@ namespace nnf
 		// Same operation order as the reference, including the sequential sum over feature maps.
 		//
 		// CACHED > 0: the column (fm_count <= CACHED) stays in registers: one read, one write. All
-		// CACHED loads are issued at once; the ones beyond fm_count re-read the last feature map
-		// (folding a value into the maximum twice changes nothing) and take no part in the sum.
+		// loads are issued at once; the registers beyond fm_count hold the maximum's starting value, which changes no
+		// maximum, and take no part in the sum. Bound by memory; a load per register, with the ones beyond fm_count
+		// re-reading the last feature map, costs the memory pipeline as much as a useful one: 16 x 21 feature maps of
+		// 129 x 129 13.6 us with 32 loads a lane, 10.3 us with the 21 it needs and a kernel of 24 registers
+		// (17: 12.3 -> 9.2 us; 33 of 128 x 128: 15.2 -> 13.8 us, with a kernel of 48; 10, four positions a lane: 16.5 -> 14.7 us).
 		// CACHED == 0: three passes in batches of eight feature maps (eight loads in flight per lane),
 		// expf values parked in the output like the reference does; a lane re-reads only what it wrote.
 		constexpr int softmax_column_batch = 8;
+
+		// The fewest feature maps the host gives a kernel of CACHED registers. What is always there needs no guard, and a
+		// launch that only waits for its own latencies ends earlier without (2 x 21 feature maps of 129 x 129: 4.3 -> 3.9 us).
+		// In the streaming kernels every access keeps its guard: a wavefront whose requests come a few instructions apart
+		// is served faster than one that sends them in one burst (16 x 21 of 129 x 129: 11.8 us without, 10.3 with;
+		// 16 x 64 of 128 x 128: 26.1 and 24.0).
+		constexpr int softmax_columns_at_least(int cached)
+		{
+			return (cached <= 2) ? 1 : (cached <= 4) ? 3 : (cached <= 8) ? 5 : (cached <= 16) ? 9 : (cached <= 24) ? 17 : (cached <= 32) ? 25 : (cached <= 48) ? 33 : 49;
+		}
 
 		template<int CACHED, bool STREAMING = false>
 		__global__ void __launch_bounds__(256) softmax_columns_kernel(float* out, const float* in, uint32_t columns, uint32_t fm_count, uint32_t plane)
@@ -277,13 +290,18 @@ namespace nnf
 			{
 				constexpr int COUNT = CACHED > 0 ? CACHED : softmax_column_batch;
 				constexpr int B = COUNT < softmax_column_batch ? COUNT : softmax_column_batch;
+				constexpr int LEAST = STREAMING ? 0 : softmax_columns_at_least(COUNT);
 				static_assert(COUNT % B == 0, "whole batches");
 				float v[COUNT];
 				#pragma unroll
 				for(int c = 0; c < COUNT; ++c)
 				{
-					const float* from = src + static_cast<size_t>(min(static_cast<uint32_t>(c), last)) * plane;
-					v[c] = STREAMING ? __builtin_nontemporal_load(from) : *from;
+					v[c] = softmax_max_init;
+					if ((c < LEAST) || (static_cast<uint32_t>(c) < fm_count)) // uniform
+					{
+						const float* from = src + static_cast<size_t>(c) * plane;
+						v[c] = STREAMING ? __builtin_nontemporal_load(from) : *from;
+					}
 				}
 				float m = softmax_max_init;
 				#pragma unroll
@@ -293,7 +311,7 @@ namespace nnf
 				#pragma unroll
 				for(int c0 = 0; c0 < COUNT; c0 += B)
 				{
-					if (static_cast<uint32_t>(c0) < fm_count) // uniform
+					if ((c0 < LEAST) || (static_cast<uint32_t>(c0) < fm_count)) // uniform
 					{
 						float x[B], e[B];
 						#pragma unroll
@@ -304,7 +322,7 @@ namespace nnf
 						for(int i = 0; i < B; ++i)
 						{
 							v[c0 + i] = e[i];
-							if (static_cast<uint32_t>(c0 + i) < fm_count) // uniform
+							if ((c0 + i < LEAST) || (static_cast<uint32_t>(c0 + i) < fm_count)) // uniform
 								sum += e[i];
 						}
 					}
@@ -313,7 +331,7 @@ namespace nnf
 				#pragma unroll
 				for(int c = 0; c < COUNT; ++c)
 				{
-					if (static_cast<uint32_t>(c) < fm_count) // uniform
+					if ((c < LEAST) || (static_cast<uint32_t>(c) < fm_count)) // uniform
 					{
 						if (STREAMING)
 							__builtin_nontemporal_store(v[c] * mult, dst + static_cast<size_t>(c) * plane);
@@ -387,7 +405,6 @@ namespace nnf
 			const size_t base = static_cast<size_t>(entry) * fm_count * plane + pos;
 			const float* src = in + base;
 			float* dst = out + base;
-			const uint32_t last = fm_count - 1;
 
 			stage_exp2_table(lds_exp);
 			__syncthreads();
@@ -399,7 +416,9 @@ namespace nnf
 			#pragma unroll
 			for(int c = 0; c < CACHED; ++c)
 			{
-				const floatx4 t = load_stream(reinterpret_cast<const floatx4*>(src + static_cast<size_t>(min(static_cast<uint32_t>(c), last)) * plane));
+				floatx4 t = { softmax_max_init, softmax_max_init, softmax_max_init, softmax_max_init };
+				if (static_cast<uint32_t>(c) < fm_count) // uniform
+					t = load_stream(reinterpret_cast<const floatx4*>(src + static_cast<size_t>(c) * plane));
 				v[c][0] = t.x; v[c][1] = t.y; v[c][2] = t.z; v[c][3] = t.w;
 			}
 			float m[4] = { softmax_max_init, softmax_max_init, softmax_max_init, softmax_max_init };
@@ -757,8 +776,12 @@ namespace nnf
 				launch_columns_kernel<8>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
 			else if (feature_map_count <= 16)
 				launch_columns_kernel<16>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
+			else if (feature_map_count <= 24)
+				launch_columns_kernel<24>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
 			else if (feature_map_count <= 32)
 				launch_columns_kernel<32>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
+			else if (feature_map_count <= 48)
+				launch_columns_kernel<48>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
 			else if (feature_map_count <= 64)
 				launch_columns_kernel<64>(stream, grid, block, output, input, columns, feature_map_count, neuron_count_per_feature_map);
 			else

@@ -747,7 +747,10 @@ def test_softmax_rows(gpu, n, c):
 @pytest.mark.parametrize("n,c,plane", [(2, 1, 5), (2, 2, 777), (2, 3, 2), (3, 4, 130), (1, 10, 49), (3, 16, 5), (2, 17, 64), (2, 21, 1000),
                                        (3, 33, 300), (2, 64, 129), (1, 1100, 70001), (4, 5, 4096),
                                        # four positions per lane (plane a multiple of 4, at least 262144 columns, up to 16 feature maps)
-                                       (1, 2, 262144), (1, 3, 262148), (2, 8, 131072), (1, 16, 262144), (1, 17, 262144)])
+                                       (1, 2, 262144), (1, 3, 262148), (2, 8, 131072), (1, 16, 262144), (1, 17, 262144),
+                                       # the last of each register count and the first of the next, in small tensors and in streaming ones (2 M floats and more)
+                                       (1, 24, 65), (1, 25, 65), (1, 32, 65), (1, 48, 65), (1, 49, 65), (1, 9, 262147), (1, 24, 90001), (1, 25, 90001),
+                                       (1, 32, 70001), (1, 48, 50001), (1, 49, 50001), (1, 64, 40001), (2, 5, 262148), (1, 9, 262148), (1, 12, 262148)])
 def test_softmax_columns_bit_exact(gpu, n, c, plane):
     """One lane per column (up to 64 feature maps, or columns too many and too long for the shared-out
     kernel): the reference's own left-to-right sum, so the bits are the oracle's."""
