@@ -620,10 +620,16 @@ namespace nnf
 		}
 
 		// Few rows cannot fill the machine with one wavefront each, and what a launch then costs is
-		// the serial work of a lane (one expf chain per value it holds): below this row count a row is
-		// spread over as many lanes as it has vectors. Measured on 256 rows of 1000 floats: 3.1 us
-		// with 256 lanes per row against 4.3 us with one wavefront per row.
+		// the serial work of a lane (one expf chain per value it holds): below few_rows a row is
+		// spread over as many lanes as it has vectors, below spread_rows over up to 1024. Measured on 256 rows of 1000
+		// floats: 3.1 us with 256 lanes per row against 4.3 us with one wavefront per row.
+		// From spread_rows on 256 lanes and several vectors each do for a long row: four wavefronts that meet at the two
+		// barriers wait less for each other than sixteen, and a compute unit holds eight rows instead of two (256 and 1024
+		// lanes: 2048 rows of 4000 11.4 and 15.6 us, 2048 of 1025 6.3 and 11.8, 4000 of 1501 12.7 and 24.0, 600 of 5000 7.4
+		// and 8.2; below spread_rows 256 of 5000 5.5 and 4.4, 64 of 8000 6.1 and 4.0). Where a wavefront holds a row
+		// by itself it stays the faster of the two (4000 of 2000 11.7 us, 13.7 with 256 lanes; 8192 of 1001 13.9 and 18.1).
 		constexpr uint32_t few_rows = 2048;
+		constexpr uint32_t spread_rows = 512;
 
 		// Columns (neuron_count_per_feature_map > 1) of more than 64 feature maps are shared out over
 		// the lanes of a workgroup: always when the workgroup's values fit this much LDS (they are
@@ -636,7 +642,7 @@ namespace nnf
 		bool try_launch_rows(hipStream_t stream, float* out, const float* in, uint32_t rows, uint32_t fm_count)
 		{
 			const uint32_t vectors = (fm_count + W - 1) / W;
-			if ((rows < few_rows) && (vectors > wave_size) && (vectors <= 1024))
+			if ((rows < few_rows) && (vectors > wave_size) && (vectors <= ((rows < spread_rows) ? 1024u : 256u)))
 			{
 				if (vectors <= 128)
 					launch_one_vector_per_lane<128, W>(stream, out, in, rows, fm_count);
@@ -655,9 +661,19 @@ namespace nnf
 			}
 			// (single floats - rows that are no multiple of four floats long, 1001 classes - up to sixteen per lane: a
 			// wavefront per row and no barrier, 8192 rows of 1001 37.5 us as one workgroup of 1024 lanes per row)
-			if (vectors <= wave_size * ((W == 1) ? 16 : 8))
+			if ((vectors <= wave_size * ((W == 1) ? 16 : 8)) && ((rows >= few_rows) || (vectors <= wave_size)))
 			{
 				launch_rows<wave_size, W>(stream, out, in, rows, fm_count, (vectors + wave_size - 1) / wave_size);
+				return true;
+			}
+			if ((rows >= spread_rows) && (vectors <= 256 * ((W == 1) ? 16 : 8)))
+			{
+				launch_rows<256, W>(stream, out, in, rows, fm_count, (vectors + 255) / 256);
+				return true;
+			}
+			if ((rows >= spread_rows) && (W == 1) && (vectors <= 512 * 16))
+			{
+				launch_rows<512, W>(stream, out, in, rows, fm_count, (vectors + 511) / 512);
 				return true;
 			}
 			if (vectors <= 1024 * 8)

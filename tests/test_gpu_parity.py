@@ -732,7 +732,10 @@ def test_argument_errors(gpu):
                                  # many rows that are no multiple of four floats long: a wavefront per row, up to sixteen floats per lane
                                  (2048, 1001), (2100, 1023), (2049, 513), (2500, 999), (4099, 1021), (2048, 1025), (3000, 130),
                                  # 4096 rows or more of up to 32 vectors: four rows to a wavefront
-                                 (4096, 100), (4097, 128), (5000, 10), (4500, 31), (4100, 33), (4099, 1), (4111, 5), (70000, 100), (4096, 124)])
+                                 (4096, 100), (4097, 128), (5000, 10), (4500, 31), (4100, 33), (4099, 1), (4111, 5), (70000, 100), (4096, 124),
+                                 # long rows: 1024 lanes each up to 511 rows, from 512 on 256 lanes (single floats beyond 4096: 512 lanes)
+                                 (511, 1028), (512, 1028), (511, 2500), (512, 2500), (2047, 4096), (512, 257), (511, 257), (2048, 2052), (600, 8192),
+                                 (512, 8196), (512, 1025), (2048, 4095), (512, 4097), (511, 4097), (512, 8191), (512, 8193), (700, 9001)])
 def test_softmax_rows(gpu, n, c):
     gen = T.rng(13, n * 100000 + c)
     x = T.normal(gen, (n, c, 1), 4.0)
