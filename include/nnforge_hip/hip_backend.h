@@ -40,7 +40,12 @@ namespace nnforge
 			typedef std::shared_ptr<const hip_linear_buffer_device> const_ptr;
 
 			explicit hip_linear_buffer_device(size_t size);
+			// `size` bytes of another allocation, from `offset` on; keeps that allocation. Many buffers that come and go
+			// together are parts of one allocation: the driver takes a quarter of a millisecond to free one, whatever its size.
+			hip_linear_buffer_device(ptr whole, size_t offset, size_t size);
 			~hip_linear_buffer_device();
+			static constexpr size_t part_alignment = 256;
+			static size_t aligned_part_size(size_t size) { return (size + part_alignment - 1) / part_alignment * part_alignment; }
 			operator void *() { return buf; }
 			operator const void *() const { return buf; }
 			operator float *() { return static_cast<float *>(buf); }
@@ -52,6 +57,7 @@ namespace nnforge
 			hip_linear_buffer_device& operator =(const hip_linear_buffer_device&) = delete;
 			void * buf;
 			size_t size;
+			ptr whole; // the allocation this buffer is a part of, if it is one
 		};
 
 		// Device selection and memory budget (nnforge/cuda/cuda_running_configuration.h)
@@ -344,7 +350,7 @@ namespace nnforge
 			// streams, device buffers for packets of `packet` entries (data and output layers once per I/O slot), pinned
 			// staging, weight pointers; what the run before left is used again when it was made for the same sizes
 			// (staging_slot_count <= 0: as many as slot_count)
-			run_buffers& prepare_run(unsigned int packet, int slot_count, bool with_output_staging, bool stats_on_device, int staging_slot_count = 0);
+			run_buffers& prepare_run(unsigned int packet, int slot_count, bool with_input_staging, bool with_output_staging, bool stats_on_device, int staging_slot_count = 0);
 			std::unique_ptr<impl> p;
 			std::unique_ptr<run_buffers> kept_run; // released when the weights, the shapes or the packet size change
 			hip_running_configuration::const_ptr hip_config;

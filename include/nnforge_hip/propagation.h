@@ -52,6 +52,10 @@ namespace nnforge
 		virtual bool read(unsigned int entry_id, const std::map<std::string, float *>& data_map) = 0;
 		virtual void set_epoch(unsigned int epoch_id) {}
 		virtual int get_entry_count() const { return -1; } // -1: unknown
+		// Where a layer's get_entry_count() entries lie in memory, one behind the other, when the reader has them so and nothing
+		// changes them during a run; null (the default): they come from read(). A backend that gets every layer's entries
+		// this way need not call read().
+		virtual const float * get_entries_in_memory(const std::string& layer_name) const { return nullptr; }
 
 	protected:
 		structured_data_bunch_reader() = default;
@@ -65,6 +69,11 @@ namespace nnforge
 		virtual ~structured_data_bunch_writer() = default;
 		virtual void set_config_map(const std::map<std::string, layer_configuration_specific> config_map) = 0;
 		virtual void write(unsigned int entry_id, const std::map<std::string, const float *>& data_map) = 0;
+		// Where a run may leave the first entry_count entries of a layer, one behind the other, when the writer has memory for
+		// them; null (the default): they go through write(). A backend that gets a place for every layer's entries need not
+		// call write(); it says which entries are there with entries_written_to_memory().
+		virtual float * get_place_for_entries(const std::string& layer_name, unsigned int entry_count) { return nullptr; }
+		virtual void entries_written_to_memory(unsigned int first_entry_id, unsigned int entry_count) {}
 
 	protected:
 		structured_data_bunch_writer() = default;
@@ -79,6 +88,8 @@ namespace nnforge
 		std::map<std::string, layer_configuration_specific> get_config_map() const override { return config_map; }
 		bool read(unsigned int entry_id, const std::map<std::string, float *>& data_map) override;
 		int get_entry_count() const override { return static_cast<int>(entry_count); }
+		// (a derived class may read differently: for its objects the answer is null unless it says otherwise itself)
+		const float * get_entries_in_memory(const std::string& layer_name) const override;
 
 	private:
 		unsigned int entry_count;

@@ -153,6 +153,18 @@ namespace
 				entries_written[dst.first] = std::max(entries_written[dst.first], entry_id + 1);
 			}
 		}
+		float * get_place_for_entries(const std::string& layer_name, unsigned int entry_count) override
+		{
+			const nnf_backend_output * const dst = by_name.at(layer_name).second;
+			// (too small: write() says so, when it comes to the entry that does not fit)
+			return (static_cast<size_t>(entry_count) * config_map.at(layer_name).get_neuron_count() <= dst->capacity_floats) ? dst->data : nullptr;
+		}
+		void entries_written_to_memory(unsigned int first_entry_id, unsigned int entry_count) override
+		{
+			if (entry_count > 0)
+				for(unsigned int& written : entries_written)
+					written = std::max(written, first_entry_id + entry_count);
+		}
 		size_t written_floats(uint32_t output_index) const
 		{
 			for(const std::pair<const std::string, std::pair<uint32_t, nnf_backend_output *> >& o : by_name)

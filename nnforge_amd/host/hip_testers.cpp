@@ -30,11 +30,20 @@ namespace nnforge
 			hip_safe_call(nnf_hip_malloc(&buf, size));
 		}
 
+		hip_linear_buffer_device::hip_linear_buffer_device(ptr whole, size_t offset, size_t size)
+			: buf(static_cast<char *>(whole->buf) + offset), size(size), whole(whole)
+		{
+			if ((offset > whole->size) || (size > whole->size - offset))
+				throw neural_network_exception("A part of a device buffer of " + std::to_string(whole->size) + " bytes cannot start at " + std::to_string(offset) + " and be " + std::to_string(size) + " bytes long");
+		}
+
 		hip_linear_buffer_device::~hip_linear_buffer_device()
 		{
-			if (buf != nullptr)
+			if ((buf != nullptr) && !whole)
 				nnf_hip_free(buf);
 		}
+
+		constexpr size_t hip_linear_buffer_device::part_alignment;
 
 		constexpr int hip_running_configuration::default_kernel_stream_count;
 
@@ -145,13 +154,28 @@ namespace nnforge
 			std::vector<hip_linear_buffer_device::const_ptr> res;
 			if (!host_data)
 				return res;
+			// the chunks of a layer as parts of one allocation, uploaded in one copy (212 chunks of 53 batch normalisation layers,
+			// each on its own: 4.0 ms)
+			size_t total = 0;
+			for(const std::vector<float>& chunk : *host_data)
+				total += hip_linear_buffer_device::aligned_part_size(chunk.size() * sizeof(float));
+			std::vector<char> packed(total);
+			size_t offset = 0;
+			for(const std::vector<float>& chunk : *host_data)
+			{
+				if (!chunk.empty())
+					std::memcpy(packed.data() + offset, chunk.data(), chunk.size() * sizeof(float));
+				offset += hip_linear_buffer_device::aligned_part_size(chunk.size() * sizeof(float));
+			}
+			hip_linear_buffer_device::ptr whole(new hip_linear_buffer_device(total));
+			if (total > 0)
+				hip_safe_call(nnf_hip_memcpy_h2d(*whole, packed.data(), total, nullptr));
+			offset = 0;
 			for(const std::vector<float>& chunk : *host_data)
 			{
 				const size_t bytes = chunk.size() * sizeof(float);
-				hip_linear_buffer_device::ptr buf(new hip_linear_buffer_device(bytes));
-				if (bytes > 0)
-					hip_safe_call(nnf_hip_memcpy_h2d(*buf, chunk.data(), bytes, nullptr));
-				res.push_back(buf);
+				res.push_back(hip_linear_buffer_device::const_ptr(new hip_linear_buffer_device(whole, offset, bytes)));
+				offset += hip_linear_buffer_device::aligned_part_size(bytes);
 			}
 			return res;
 		}

@@ -11,6 +11,7 @@
 #include <fstream>
 #include <mutex>
 #include <thread>
+#include <typeinfo>
 
 #include <sched.h>
 
@@ -104,6 +105,14 @@ namespace nnforge
 			std::memcpy(dst.second, src->second + static_cast<size_t>(entry_id) * neuron_count, neuron_count * sizeof(float));
 		}
 		return true;
+	}
+
+	const float * memory_data_bunch_reader::get_entries_in_memory(const std::string& layer_name) const
+	{
+		if (typeid(*this) != typeid(memory_data_bunch_reader))
+			return nullptr;
+		const std::map<std::string, const float *>::const_iterator src = data.find(layer_name);
+		return (src != data.end()) ? src->second : nullptr;
 	}
 
 	void memory_data_bunch_writer::set_config_map(const std::map<std::string, layer_configuration_specific> new_config_map)

@@ -420,6 +420,42 @@ def test_inference_from_data_set_files_to_data_set_files(tmp_path):
         backend.run_dataset(S.schema_text(layers), weights, {"images": tmp_path / "nowhere.dt"}, outputs)
 
 
+@pytest.mark.parametrize("n,c,side,options", [
+    (1, 3, 5, {}), (2, 1, 1, {}),                       # one small copy, by the calling thread
+    (1, 64, 91, {}), (1, 64, 90, {"host_thread_count": 1}),  # just above and below what several threads share out
+    (3, 65, 151, {}),                                   # several pieces, the last of them short
+    (7, 40, 129, {"max_entry_count": 3}),               # packets, the last of them short
+    (6, 40, 129, {"max_entry_count": 3, "kernel_stream_count": 3, "one_launch_per_group": True}),
+    (5, 16, 64, {"max_entry_count": 5, "profile": True}),
+])
+def test_entries_in_the_callers_arrays_and_in_files_give_the_same(tmp_path, n, c, side, options):
+    """run_schema copies straight between the caller's arrays and the device, run_dataset goes entry by entry through pinned
+    staging: the same bits, and the oracle's; a place that is too small is the same error as before."""
+    from nnforge_amd import schemas
+
+    gen = T.rng(71, n * 1000 + side)
+    x, y = (T.normal(gen, (n, c, side, side), 1.0) for _ in range(2))
+    bn = [T.normal(gen, (c,), 0.3) for _ in range(3)] + [gen.random(c, dtype=F32) + F32(0.5)]
+    L = schemas.L
+    layers = [L("Data", "x"), L("Data", "y"), L("BatchNorm", "bn", ["x"], feature_map_count=c), L("ReLU", "relu", ["bn"]), L("Add", "sum", ["relu", "y"])]
+    weights, inputs, outputs = {"bn": bn}, {"x": x, "y": y}, {"relu": (n, c, side, side), "sum": (n, c, side, side)}
+    got, rep = backend.run_schema(S.schema_text(layers), weights, inputs, outputs, **options)
+    assert rep["entries"] == n
+    relu = oracle.rectified_linear(oracle.batch_norm(x.reshape(n, c, -1), *bn))
+    assert_bits(got["relu"].reshape(n, c, -1), relu, "relu")
+    assert_bits(got["sum"].reshape(n, c, -1), oracle.add([relu, y.reshape(n, c, -1)]), "sum")
+    for name, a in inputs.items():
+        backend.write_dataset(tmp_path / (name + ".dt"), a)
+    paths = {name: tmp_path / (name + ".dt") for name in list(inputs) + list(outputs)}
+    backend.run_dataset(S.schema_text(layers), weights, {k: paths[k] for k in inputs}, {k: paths[k] for k in outputs},
+                        **{k: v for k, v in options.items() if k != "profile"})
+    for name in outputs:
+        assert_bits(backend.read_dataset(paths[name]), got[name], name + " through files")
+    with pytest.raises(backend.BackendError, match="Output buffer for layer sum is too small"):
+        backend.run_schema(S.schema_text(layers), weights, inputs, {"relu": outputs["relu"], "sum": (n, c, side, side - 1)} if side > 1 else
+                           {"relu": outputs["relu"], "sum": (n - 1, c, side, side)}, **options)
+
+
 @pytest.mark.parametrize("mode", ["together", "streams", "plain"])
 def test_resnet50_post_convolution_graph_layer_by_layer(mode):
     """Config 4 through the driver at a small entry count: every output of the 50 steps (48 groups, the last block's group
