@@ -315,8 +315,8 @@ namespace nnf
 					{
 						float x[B], e[B];
 						#pragma unroll
-						for(int i = 0; i < B; ++i)
-							x[i] = v[c0 + i] - m;
+						for(int i = 0; i < B; ++i) // (a zero keeps a batch that is not full off the branch for large arguments)
+							x[i] = ((c0 + i < LEAST) || (static_cast<uint32_t>(c0 + i) < fm_count)) ? v[c0 + i] - m : 0.0f;
 						nnf_expf_batch<B>(x, e, exp_ctx);
 						#pragma unroll
 						for(int i = 0; i < B; ++i)
@@ -461,7 +461,114 @@ namespace nnf
 			}
 		}
 
-		// neuron_count_per_feature_map > 1 and more than 64 feature maps: one lane per column would make
+		// neuron_count_per_feature_map > 1 and 65 to 1024 feature maps: a workgroup of BLOCK lanes takes P consecutive columns
+		// and holds them in registers: lane (slice, position) the feature maps slice, slice + S, ... of its position, S =
+		// BLOCK / P, up to VALUES of them. All loads are requested at once, one read and one write of memory; maximum and sum
+		// are combined through LDS in slice order. The maximum is the reference's; the sum is S partial sums added in order, so
+		// results can differ from the reference in the last bits (bar: 1e-5 relative, as for rows).
+		// Bound by memory. With the values in LDS and slices of contiguous feature maps walked eight loads at a time (the kernel
+		// below) a launch waited for batch after batch: 2 x 683 feature maps of 18 x 18 11.1 us, 6.3 this way; 128 entries of 200
+		// of 28 x 28 45.1 and 36.6; 8 of 300 of 128 x 128 85.4 and 65.1; 8 of 80 of 192 x 192 45.8 and 38.3.
+		// What the host chooses by columns and feature maps: many columns - a whole wavefront along the positions, streaming
+		// accesses; few - 16 positions, or 8, that leave more workgroups. The shapes beside each other in its comments.
+		template<int BLOCK, int P, int VALUES, bool STREAMING>
+		__global__ void __launch_bounds__(BLOCK) softmax_columns_shared_kernel(float* out, const float* in, uint32_t columns, uint32_t fm_count, uint32_t plane)
+		{
+			constexpr uint32_t S = BLOCK / P;
+			constexpr int B = softmax_column_batch;
+			static_assert((VALUES % B == 0) && (S <= 64), "whole batches; every slice has a feature map");
+			__shared__ uint64_t lds_exp[exp_lds_entries];
+			__shared__ float lds_partial[2][S][P];
+			const uint32_t p = threadIdx.x % P;
+			const uint32_t slice = (P >= wave_size) ? __builtin_amdgcn_readfirstlane(threadIdx.x / P) : threadIdx.x / P;
+			// neighbouring blocks of positions lie in the same cache lines: sixteen of them to workgroups of one XCD
+			const uint32_t column = xcd_grouped(blockIdx.x, 16u, gridDim.x) * P + p;
+			const bool valid = column < columns;
+			const uint32_t col = valid ? column : columns - 1; // lanes past the end shadow the last column and store nothing
+			const uint32_t entry = col / plane;
+			const uint32_t pos = col - entry * plane;
+			const size_t base = static_cast<size_t>(entry) * fm_count * plane + static_cast<size_t>(slice) * plane + pos;
+			const float* src = in + base;
+			float* dst = out + base;
+			const uint32_t rounds = (fm_count + S - 1) / S; // feature maps of a slice; the last round is not there for every slice
+			const size_t step = static_cast<size_t>(S) * plane;
+
+			float v[VALUES];
+			#pragma unroll
+			for(int i = 0; i < VALUES; ++i)
+			{
+				v[i] = softmax_max_init;
+				if (static_cast<uint32_t>(i) < rounds) // uniform
+				{
+					// a slice that has no feature map in the last round takes its first one again: no other maximum
+					const float* from = src + ((i * S + slice < fm_count) ? i * step : 0);
+					v[i] = STREAMING ? __builtin_nontemporal_load(from) : *from;
+				}
+			}
+			stage_exp2_table(lds_exp);
+			__syncthreads();
+			const exp_context exp_ctx = exp_context_from_lds(lds_exp);
+
+			float m = softmax_max_init;
+			#pragma unroll
+			for(int i = 0; i < VALUES; ++i)
+				m = ref_max(m, v[i]);
+			lds_partial[0][slice][p] = m;
+			__syncthreads();
+			m = softmax_max_init;
+			#pragma unroll 16
+			for(uint32_t s = 0; s < S; ++s)
+				m = ref_max(m, lds_partial[0][s][p]);
+
+			float sum = 0.0f;
+			#pragma unroll
+			for(int i0 = 0; i0 < VALUES; i0 += B)
+			{
+				if (static_cast<uint32_t>(i0) < rounds) // uniform
+				{
+					float x[B], e[B];
+					#pragma unroll
+					for(int i = 0; i < B; ++i)
+						x[i] = (static_cast<uint32_t>(i0 + i) < rounds) ? v[i0 + i] - m : 0.0f;
+					nnf_expf_batch<B>(x, e, exp_ctx);
+					#pragma unroll
+					for(int i = 0; i < B; ++i)
+					{
+						v[i0 + i] = e[i];
+						sum += ((i0 + i) * S + slice < fm_count) ? e[i] : 0.0f;
+					}
+				}
+			}
+			lds_partial[1][slice][p] = sum;
+			__syncthreads();
+			sum = 0.0f;
+			#pragma unroll 16
+			for(uint32_t s = 0; s < S; ++s)
+				sum += lds_partial[1][s][p];
+
+			const float mult = 1.0f / sum;
+			if (!valid)
+				return;
+			#pragma unroll
+			for(int i = 0; i < VALUES; ++i)
+			{
+				if ((static_cast<uint32_t>(i) < rounds) && (i * S + slice < fm_count))
+				{
+					if (STREAMING)
+						__builtin_nontemporal_store(v[i] * mult, dst + i * step);
+					else
+						dst[i * step] = v[i] * mult;
+				}
+			}
+		}
+
+		template<int BLOCK, int P, int VALUES, bool STREAMING>
+		void launch_columns_shared(hipStream_t stream, float* out, const float* in, uint32_t columns, uint32_t fm_count, uint32_t plane)
+		{
+			NNF_LAUNCH((softmax_columns_shared_kernel<BLOCK, P, VALUES, STREAMING>), dim3((columns + P - 1) / P), dim3(BLOCK), 0, stream, out, in, columns, fm_count, plane);
+		}
+
+		// neuron_count_per_feature_map > 1 and more than 1024 feature maps: one lane per column would make
 		// every lane walk a long column alone, with three passes over memory. A workgroup of 256 lanes
 		// takes P consecutive columns; the feature maps are cut into S = 256 / P contiguous slices, lane
 		// (slice, position) walks its slice in batches of eight, and the slices are combined through LDS
@@ -486,8 +593,7 @@ namespace nnf
 			const uint32_t p = threadIdx.x % P;
 			const uint32_t slice = threadIdx.x / P;
 			// Neighbouring blocks of positions lie in the same cache lines (P positions are P * 4 bytes of every feature
-			// map's row): sixteen of them (four of the wide ones) go to workgroups of one XCD, where the lines meet in one
-			// L2 (64 x 1000 feature maps of 7 x 7: 22.0 -> 17.2 us; 256 x 128 of 28 x 28: 45.8 -> 43.8 us).
+			// map's row): sixteen of them (four of the wide ones) go to workgroups of one XCD, where the lines meet in one L2.
 			const uint32_t column = xcd_grouped(blockIdx.x, (P < 32) ? 16u : 4u, gridDim.x) * P + p;
 			const bool valid = column < columns;
 			const uint32_t col = valid ? column : columns - 1; // lanes past the end shadow the last column and store nothing
@@ -631,10 +737,9 @@ namespace nnf
 		constexpr uint32_t few_rows = 2048;
 		constexpr uint32_t spread_rows = 512;
 
-		// Columns (neuron_count_per_feature_map > 1) of more than 64 feature maps are shared out over
-		// the lanes of a workgroup: always when the workgroup's values fit this much LDS (they are
-		// then read from memory once), otherwise up to this many columns (small tensors, re-read from
-		// the caches); beyond both, one lane walks a column in three passes.
+		// Columns (neuron_count_per_feature_map > 1) of more than 1024 feature maps are shared out over the lanes of a workgroup
+		// up to this many columns: from LDS when eight positions' values fit this much of it (read from memory once), otherwise
+		// re-read from the caches; beyond that, one lane walks a column in three passes.
 		constexpr size_t staged_bytes_limit = 60 * 1024;
 		constexpr uint32_t sliced_columns_limit = 65536;
 
@@ -718,45 +823,16 @@ namespace nnf
 		else
 		{
 			const uint32_t columns = entry_count * neuron_count_per_feature_map;
-			if (feature_map_count > 64)
+			if (feature_map_count > 1024)
 			{
-				// a whole wavefront along the positions (256-byte accesses) once that still gives every
-				// compute unit a few workgroups; fewer positions when that is what lets the values fit LDS
-				uint32_t positions = (columns >= 64u * 512u) ? 64u : 16u;
-				// half a wavefront along the positions when that lets a compute unit hold twice the workgroups
-				// (256 x 128 feature maps of 28 x 28: 52.7 us with 64 positions and 32 KB, 46.3 us with 32)
-				if ((positions == 64u) && (static_cast<size_t>(feature_map_count) * positions * sizeof(float) > 24u * 1024u))
-					positions = 32u;
-				while ((positions > 16u) && (static_cast<size_t>(feature_map_count) * positions * sizeof(float) > staged_bytes_limit))
-					positions /= 2;
-				// eight positions for small tensors whose values then fit: 1000 feature maps of 7 x 7 in one read and one
-				// write, 22 us for 64 entries against 36 us in three passes with sixteen (large tensors: 32-byte accesses
-				// cost more than the passes, 315 against 137 us on 32 x 150 feature maps of 128 x 128)
-				if ((positions == 16u) && (columns <= sliced_columns_limit)
-					&& (static_cast<size_t>(feature_map_count) * 16u * sizeof(float) > staged_bytes_limit)
-					&& (static_cast<size_t>(feature_map_count) * 8u * sizeof(float) <= staged_bytes_limit))
-					positions = 8u;
-				const size_t staged_bytes = static_cast<size_t>(feature_map_count) * positions * sizeof(float);
-				const dim3 sliced_grid((columns + positions - 1) / positions);
-				if (staged_bytes <= staged_bytes_limit)
-				{
-					if (positions == 64)
-						NNF_LAUNCH((softmax_columns_sliced_kernel<64, true>), sliced_grid, dim3(256), staged_bytes, stream,
-							output, input, columns, feature_map_count, neuron_count_per_feature_map);
-					else if (positions == 32)
-						NNF_LAUNCH((softmax_columns_sliced_kernel<32, true>), sliced_grid, dim3(256), staged_bytes, stream,
-							output, input, columns, feature_map_count, neuron_count_per_feature_map);
-					else if (positions == 16)
-						NNF_LAUNCH((softmax_columns_sliced_kernel<16, true>), sliced_grid, dim3(256), staged_bytes, stream,
-							output, input, columns, feature_map_count, neuron_count_per_feature_map);
-					else
-						NNF_LAUNCH((softmax_columns_sliced_kernel<8, true>), sliced_grid, dim3(256), staged_bytes, stream,
-							output, input, columns, feature_map_count, neuron_count_per_feature_map);
-					return launch_status();
-				}
+				// eight positions where the values then fit LDS: one read and one write; otherwise three passes
+				const size_t staged_bytes = static_cast<size_t>(feature_map_count) * 8u * sizeof(float);
 				if (columns <= sliced_columns_limit)
 				{
-					if (columns >= 64u * 512u)
+					if (staged_bytes <= staged_bytes_limit)
+						NNF_LAUNCH((softmax_columns_sliced_kernel<8, true>), dim3((columns + 7) / 8), dim3(256), staged_bytes, stream,
+							output, input, columns, feature_map_count, neuron_count_per_feature_map);
+					else if (columns >= 64u * 512u)
 						NNF_LAUNCH((softmax_columns_sliced_kernel<64, false>), dim3((columns + 63) / 64), dim3(256), 0, stream,
 							output, input, columns, feature_map_count, neuron_count_per_feature_map);
 					else
@@ -764,6 +840,40 @@ namespace nnf
 							output, input, columns, feature_map_count, neuron_count_per_feature_map);
 					return launch_status();
 				}
+			}
+			else if (feature_map_count > 64)
+			{
+				// the fewest registers that hold a column; both sides of each line measured:
+				const uint32_t plane = neuron_count_per_feature_map;
+				if (feature_map_count <= 128)
+				{
+					if (columns >= 20480u) // 32 x 100 of 28 x 28 7.1 us, 7.5 with 16 positions; 2 x 66 of 64 x 64 4.7 and 3.9
+						launch_columns_shared<512, 64, 16, true>(stream, output, input, columns, feature_map_count, plane);
+					else
+						launch_columns_shared<256, 16, 8, false>(stream, output, input, columns, feature_map_count, plane);
+				}
+				else if (feature_map_count <= 256)
+				{
+					if (columns >= 81920u) // 8 x 150 of 128 x 128 34.2 us, 39.2 with 16 positions; 64 x 200 of 28 x 28 20.0 and 17.6
+						launch_columns_shared<512, 64, 32, true>(stream, output, input, columns, feature_map_count, plane);
+					else
+						launch_columns_shared<256, 16, 16, false>(stream, output, input, columns, feature_map_count, plane);
+				}
+				else if (feature_map_count <= 512)
+				{
+					if (columns >= 32768u) // 16 x 400 of 64 x 64 41.6 us, 48.4 with 16 positions; 2 x 500 of 100 x 100 21.3 and 17.3
+						launch_columns_shared<512, 64, 64, true>(stream, output, input, columns, feature_map_count, plane);
+					else
+						launch_columns_shared<512, 16, 16, false>(stream, output, input, columns, feature_map_count, plane);
+				}
+				else
+				{
+					if (columns >= 4352u) // 32 x 600 of 28 x 28 34.7 us, 41.8 with 8 positions; 4 x 1000 of 33 x 33 15.2 and 14.8
+						launch_columns_shared<512, 16, 32, false>(stream, output, input, columns, feature_map_count, plane);
+					else
+						launch_columns_shared<512, 8, 16, false>(stream, output, input, columns, feature_map_count, plane);
+				}
+				return launch_status();
 			}
 			// few columns: one wavefront per workgroup spreads them over more compute units
 			const uint32_t block_size = (columns >= 256u * 1024u) ? 256u : 64u;

@@ -773,7 +773,12 @@ def test_softmax_columns_bit_exact(gpu, n, c, plane):
                                        (1, 300, 65536), (1, 300, 65537), (1, 480, 33000), (1, 481, 33000),
                                        # up to 65536 columns: 8 positions x up to 1920 feature maps staged; 32 positions from 97 feature maps on in large tensors
                                        (64, 1000, 49), (2, 1920, 70), (2, 1921, 70), (3, 1500, 9), (1, 1100, 65536),
-                                       (1, 96, 33000), (1, 97, 33000), (2, 128, 20000)])
+                                       (1, 96, 33000), (1, 97, 33000), (2, 128, 20000),
+                                       # values held in registers, up to 1024 feature maps: both sides of every line the host draws, whole and short last
+                                       # rounds of a slice, whole and short last workgroups
+                                       (1, 65, 20479), (1, 65, 20480), (1, 65, 20481), (1, 128, 20480), (3, 128, 21), (1, 129, 81919), (1, 129, 81920),
+                                       (1, 256, 81921), (2, 256, 40), (1, 257, 32767), (1, 257, 32769), (1, 512, 32768), (5, 512, 13), (1, 513, 4351),
+                                       (1, 513, 4353), (1, 1024, 4352), (2, 1024, 17), (1, 1025, 33), (1, 1023, 66000)])
 def test_softmax_columns_sliced(gpu, n, c, plane):
     """More than 64 feature maps: a column is shared out over 4 to 32 lanes whose partial sums are
     added in slice order, so the bar is the one stated for softmax, 1e-5 relative."""
