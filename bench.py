@@ -1154,7 +1154,7 @@ def main():
                        "feature_map_stat": "nnf::stat_runs_kernel", "walking_grid": "nnf::chain_kernel_persistent",
                        "global_average": "nnf::global_pool_linear_kernel", "joined_global_average": "nnf::global_pool_linear_kernel",
                        "softmax_many_rows": "nnf::softmax_rows_kernel", "softmax_rows_1001": "nnf::softmax_rows_kernel", "softmax_short_rows": "nnf::softmax_rows_kernel",
-                       "softmax_columns": "nnf::softmax_columns_kernel", "softmax_wide_columns": "nnf::softmax_columns_sliced_kernel",
+                       "softmax_columns": "nnf::softmax_columns_kernel", "softmax_wide_columns": "nnf::softmax_columns_shared_kernel",
                        "inception_block": "nnf::chain_entries_batch_kernel", "inception_block_copies": "nnf::chain_batch_kernel + nnf::concat_kernel",
                        "config4": "all kernels of one pass of the launch plan (nnf::chain_batch_mixed_kernel, nnf::chain_batch_kernel, nnf::chain_kernel, nnf::global_pool_linear_kernel, nnf::softmax_rows_kernel)",
                        "config4_direct": "all kernels of one pass (nnf::chain_kernel x 49, nnf::global_pool_kernel, nnf::softmax_rows_kernel)"}.get(args.workload, "nnf::chain_kernel"),

@@ -9,8 +9,8 @@
 //    read once and written once. The sum is a fixed tree, so it can differ from the reference's
 //    left-to-right sum in the last bits.
 //  - neuron_count_per_feature_map > 1: feature maps are strided by the plane size ("columns").
-//    Lanes run along the spatial positions (coalesced), each lane walks its column in feature-map
-//    order with the reference's own sequential sum.
+//    Lanes run along the spatial positions (coalesced). Up to 64 feature maps a lane walks its column in feature-map
+//    order with the reference's own sequential sum; more of them are shared out over lanes, whose sums are added in order.
 #include "nnf_common.h"
 
 namespace nnf
